@@ -142,3 +142,17 @@ int llg_moe_gemm_enqueue(LlgDevice *d, const LlgObject *gate, const LlgObject *u
                          const LlgObject *down, int n_exp, int k, int hidden, int eff,
                          const float *d_x, int n_tok, const int32_t *ids, const float *w,
                          float *d_out, uint8_t *ws);
+// The combine, shared by both batch forms: out = the slots' weighted sum of the
+// ksplit partial products of Y.
+void llg_moe_combine_launch(hipStream_t st, const float *Y, const int32_t *pair_row, const float *w,
+                            int k, int n_tok, int hidden, int ksplit, long long ystride,
+                            float *out);
+
+// MoE batches at fp32 precision as grouped MFMA GEMMs (llg_moe_split.hip).
+bool llg_moe_split_use(const LlgObject *gate, const LlgObject *down, int hidden, int eff, int n_tok,
+                       int k, int n_exp);
+size_t llg_moe_split_ws_bytes(int cus, int n_tok, int k, int n_exp, int hidden, int eff);
+int llg_moe_split_enqueue(LlgDevice *d, const LlgObject *gate, const LlgObject *up,
+                          const LlgObject *down, int n_exp, int k, int hidden, int eff,
+                          const float *d_x, int n_tok, const int32_t *ids, const float *w,
+                          float *d_out, uint8_t *ws);

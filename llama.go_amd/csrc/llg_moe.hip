@@ -16,9 +16,10 @@
 //                  order, so results are the same on every run
 // Expert e's rows are e*eff + j of gate/up and e*hidden + d of down, the
 // addressing of ReadContiguousRows (flash/storage.go:72-94).
-// Batches of 16 or more tokens over Q4_0 experts go to the grouped MFMA GEMM
-// path (llg_moe_gemm.hip); smaller batches and other types use the kernels
-// below token by token.
+// Batches of 16 or more tokens over Q4_0 experts of wide rows go to the grouped
+// f16 GEMMs (llg_moe_gemm.hip), other batches with enough tokens per expert to
+// the grouped GEMMs at fp32 precision (llg_moe_split.hip); the rest use the
+// kernels below token by token.
 #include <algorithm>
 
 #include "llg_common.hpp"
@@ -548,6 +549,10 @@ static bool use_gemm(const MoeArgs &a, int n_tok) {
     return llg_moe_gemm_supported(a.gate->fmt.type, a.hidden, a.eff, n_tok);
 }
 
+static bool use_split(const MoeArgs &a, int n_tok) {
+    return llg_moe_split_use(a.gate, a.down, a.hidden, a.eff, n_tok, a.k, a.n_exp);
+}
+
 // Column chunks of h the decode down kernels split a row into (64 blocks for
 // the persistent form, up to MOE_DN_CHUNK for the tile form).
 static int moe_dec_chunks(const MoeArgs &a, bool persistent) {
@@ -560,10 +565,12 @@ static size_t moe_hbuf_bytes(const MoeArgs &a, int n_tok) {
     return (size_t)llg_align((long long)n_tok * a.k * a.eff * 4, 256);
 }
 
-static size_t moe_ws_bytes(const MoeArgs &a, int n_tok) {
+static size_t moe_ws_bytes(LlgDevice *d, const MoeArgs &a, int n_tok) {
     const size_t head = (size_t)llg_align((long long)n_tok * a.k * 4, 256) * 2;
     if (use_gemm(a, n_tok))
         return head + llg_moe_gemm_ws_bytes(n_tok, a.k, a.n_exp, a.hidden, a.eff);
+    if (use_split(a, n_tok))
+        return head + llg_moe_split_ws_bytes(llg_cu_count(d), n_tok, a.k, a.n_exp, a.hidden, a.eff);
     // h, then the down partials (the larger chunk count of the two forms)
     return head + moe_hbuf_bytes(a, n_tok) +
            (size_t)n_tok * a.k * moe_dec_chunks(a, true) * a.hidden * 4;
@@ -642,6 +649,9 @@ static int moe_enqueue(LlgDevice *d, const MoeArgs &a, const float *d_x, int n_t
     if (use_gemm(a, n_tok))  // batched tokens: grouped MFMA GEMMs
         return llg_moe_gemm_enqueue(d, a.gate, a.up, a.down, a.n_exp, a.k, a.hidden, a.eff, d_x,
                                     n_tok, ids, w, d_out, ws + 2 * kb);
+    if (use_split(a, n_tok))  // other batches: grouped GEMMs at fp32 precision
+        return llg_moe_split_enqueue(d, a.gate, a.up, a.down, a.n_exp, a.k, a.hidden, a.eff, d_x,
+                                     n_tok, ids, w, d_out, ws + 2 * kb);
     switch (a.gate->fmt.type) {
     case LLG_TYPE_Q4_0:
         moe_launch_experts<LLG_TYPE_Q4_0>(st, llg_cu_count(d), a, n_tok, ids, w, d_x, hbuf, part, d_out);
@@ -675,7 +685,7 @@ int llg_hipd_moe_ffn(LlgHipDevice h, int64_t hr, int64_t hg, int64_t hu, int64_t
     if (!d_x || !d_out || n_tok <= 0) return llg_set_error(d, LLG_E_ARG, "moe: bad arguments");
     if (((uintptr_t)d_x | (uintptr_t)d_out) & 15)
         return llg_set_error(d, LLG_E_ALIGN, "moe: x and out must be 16-byte aligned");
-    uint8_t *ws = (uint8_t *)llg_ws(d, moe_ws_bytes(a, n_tok), &rc);
+    uint8_t *ws = (uint8_t *)llg_ws(d, moe_ws_bytes(d, a, n_tok), &rc);
     if (rc) return rc;
     return moe_enqueue(d, a, d_x, n_tok, d_out, d_ids, d_w, ws);
 }
@@ -693,7 +703,7 @@ int llg_hip_moe_ffn(LlgHipDevice h, int64_t hr, int64_t hg, int64_t hu, int64_t 
     const long long o_ids = o_out + llg_align((long long)xb, 256);
     const long long o_w = o_ids + llg_align((long long)n_tok * k * 4, 256);
     const long long o_ws = o_w + llg_align((long long)n_tok * k * 4, 256);
-    uint8_t *ws = (uint8_t *)llg_ws(d, o_ws + moe_ws_bytes(a, n_tok), &rc);
+    uint8_t *ws = (uint8_t *)llg_ws(d, o_ws + moe_ws_bytes(d, a, n_tok), &rc);
     if (rc) return rc;
     if ((rc = llg_h2d(d, ws, x, xb))) return rc;
     rc = moe_enqueue(d, a, (const float *)ws, n_tok, (float *)(ws + o_out),

@@ -3,10 +3,11 @@
 // reference runs them one token at a time, cmd/generate.go:88-96).
 //
 //   1. k_moe_router (llg_moe.hip): ids / weights per token
-//   2. k_moe_group: counting sort of the (token, slot) pairs by expert, the
+//   2. k_moe_group_x16: counting sort of the (token, slot) pairs by expert, the
 //      pair <-> row maps, and a list of M-tiles (expert, first row, rows):
 //      each expert's rows in the fewest tiles of at most 80 rows, balanced
-//   3. k_moe_x16: X -> f16 in the MFMA K order (k_order)
+//      and, in its other workgroups,
+//   3. X -> f16 in the MFMA K order (k_order)
 //   4. k_moe_gemm<0>: G = X_e . gate_e^T, U = X_e . up_e^T on v_mfma_f32_16x16x32_f16,
 //      epilogue H = silu(G) * U (moe_forward.go:128-132) stored f16, same K order
 //   5. k_moe_gemm<1>: Y = H_e . down_e^T
@@ -34,6 +35,7 @@
 
 #include "llg_common.hpp"
 #include "llg_internal.hpp"
+#include "llg_moe_group.hpp"
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
@@ -50,57 +52,18 @@ typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 #endif
 #define GM_STORE_STEP 2           // MFMA step of a chunk before which the next A is stored
 
-// ---------------------------------------------------------------------------
-// Grouping: pairs p = t*k + s sorted by expert (order within an expert is not
-// significant: each row's result depends only on its own token).
-// tiles[i] = (expert, first row, rows); n_tiles[0] = count.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void k_moe_group(const int32_t *__restrict__ ids, int n_pairs,
-                                                    int n_exp, int32_t *__restrict__ row_pair,
-                                                    int32_t *__restrict__ pair_row,
-                                                    int4 *__restrict__ tiles,
-                                                    int32_t *__restrict__ n_tiles) {
-    __shared__ int cnt[64], off[65], fill[64];
-    const int tid = threadIdx.x;
-    if (tid < 64) {
-        cnt[tid] = 0;
-        fill[tid] = 0;
-    }
-    __syncthreads();
-    for (int p = tid; p < n_pairs; p += blockDim.x) atomicAdd(&cnt[ids[p]], 1);
-    __syncthreads();
-    if (tid == 0) {
-        int o = 0, nt = 0;
-        for (int e = 0; e < n_exp; e++) {
-            off[e] = o;
-            // the fewest tiles of at most GM_BM rows (each streams the
-            // expert's weights once), their sizes within one of each other
-            const int n = (cnt[e] + GM_BM - 1) / GM_BM;
-            for (int i = 0, r = 0; i < n; i++) {
-                const int rows = cnt[e] / n + (i < cnt[e] % n ? 1 : 0);
-                tiles[nt++] = make_int4(e, o + r, rows, 0);
-                r += rows;
-            }
-            o += cnt[e];
-        }
-        off[n_exp] = o;
-        *n_tiles = nt;
-    }
-    __syncthreads();
-    for (int p = tid; p < n_pairs; p += blockDim.x) {
-        const int e = ids[p];
-        const int r = off[e] + atomicAdd(&fill[e], 1);
-        row_pair[r] = p;
-        pair_row[p] = r;
-    }
-}
-
 // X (fp32, [n_tok x K]) -> f16 in the MFMA K order (k_order; K is a
 // multiple of 128, so chunks never straddle rows): 8-group i goes to 8-group
 // (i & ~15) | (i & 3) << 2 | (i >> 2) & 3, its elements in the order
-// [0,4,1,5,2,6,3,7].
-__global__ void k_moe_x16(const float *__restrict__ x, long long n8, _Float16 *__restrict__ x16) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;  // 8-group index
+// [0,4,1,5,2,6,3,7].  Workgroup 0 groups the pairs meanwhile (as in
+// k_moe_group_split).
+__global__ __launch_bounds__(MOE_GROUP_THREADS) void k_moe_group_x16(
+    MoeGroupArgs ga, const float *__restrict__ x, long long n8, _Float16 *__restrict__ x16) {
+    if (blockIdx.x == 0) {
+        moe_group(ga);
+        return;
+    }
+    const long long i = (blockIdx.x - 1LL) * blockDim.x + threadIdx.x;  // 8-group index
     if (i >= n8) return;
     const float4 a = reinterpret_cast<const float4 *>(x)[2 * i];
     const float4 b = reinterpret_cast<const float4 *>(x)[2 * i + 1];
@@ -426,6 +389,14 @@ static int down_split(int eff) {
     return nc % 4 == 0 ? 4 : nc % 2 == 0 ? 2 : 1;
 }
 
+void llg_moe_combine_launch(hipStream_t st, const float *Y, const int32_t *pair_row, const float *w,
+                            int k, int n_tok, int hidden, int ksplit, long long ystride,
+                            float *out) {
+    const long long n4 = (long long)n_tok * hidden / 4;
+    hipLaunchKernelGGL(k_moe_combine, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, Y,
+                       pair_row, w, k, n_tok, hidden, ksplit, ystride, out);
+}
+
 // ---------------------------------------------------------------------------
 size_t llg_moe_gemm_ws_bytes(int n_tok, int k, int n_exp, int hidden, int eff) {
     const long long np = (long long)n_tok * k;
@@ -468,11 +439,11 @@ int llg_moe_gemm_enqueue(LlgDevice *d, const LlgObject *gate, const LlgObject *u
     p += llg_align(np * eff * 2, 256);
     float *Y = reinterpret_cast<float *>(p);
 
-    hipLaunchKernelGGL(k_moe_group, dim3(1), dim3(1024), 0, st, ids, (int)np, n_exp, row_pair,
-                       pair_row, tiles, n_tiles);
     const long long n8 = (long long)n_tok * hidden / 8;
-    hipLaunchKernelGGL(k_moe_x16, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, st, d_x, n8,
-                       x16);
+    const MoeGroupArgs ga = {ids, (int)np, n_exp, GM_BM, row_pair, pair_row, tiles, n_tiles};
+    hipLaunchKernelGGL(k_moe_group_x16,
+                       dim3((unsigned)((n8 + MOE_GROUP_THREADS - 1) / MOE_GROUP_THREADS + 1)),
+                       dim3(MOE_GROUP_THREADS), 0, st, ga, d_x, n8, x16);
     hipLaunchKernelGGL((k_moe_gemm<0>), dim3((unsigned)(nt_max * (eff / (4 * gm_wave_cols<0>())))),
                        dim3(256), 0, st,
                        tiles, n_tiles, row_pair, k, x16, tg, tu, eff, hidden, eff, H,
@@ -484,9 +455,7 @@ int llg_moe_gemm_enqueue(LlgDevice *d, const LlgObject *gate, const LlgObject *u
                        dim3(256), 0, st, tiles, n_tiles, row_pair, k, H, td,
                        (const uint8_t *)nullptr, hidden, eff, hidden, (_Float16 *)nullptr, Y,
                        ksplit, ystride);
-    const long long n4 = (long long)n_tok * hidden / 4;
-    hipLaunchKernelGGL(k_moe_combine, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, Y,
-                       pair_row, w, k, n_tok, hidden, ksplit, ystride, d_out);
+    llg_moe_combine_launch(st, Y, pair_row, w, k, n_tok, hidden, ksplit, ystride, d_out);
     LLG_LAUNCH_CHECK(d, "moe grouped gemm");
     return 0;
 }
