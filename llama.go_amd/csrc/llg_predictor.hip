@@ -43,6 +43,7 @@ __global__ __launch_bounds__(256) void k_pred_hidden(const uint8_t *__restrict__
 
 // One workgroup of 256 threads per 64-neuron tile: logits, optional output,
 // and the tile's 64-bit active mask (bit i <=> logit[tile*64+i] > thr).
+template <int MV>
 __global__ __launch_bounds__(256) void k_pred_logits(const uint8_t *__restrict__ wout,
                                                      long long stride, int ff, int rank,
                                                      const float *__restrict__ partial,
@@ -53,7 +54,7 @@ __global__ __launch_bounds__(256) void k_pred_logits(const uint8_t *__restrict__
     float *hid = sh;
     float *lg = sh + ((rank + 3) & ~3);
     const int tile0 = blockIdx.x * 64;
-    WoutTile t;
+    WoutTile<MV> t;
     load_wout_tile(t, wout, stride, ff, rank, tile0);
     load_hidden<PRED_SPLIT>(hid, partial, rank);
     __syncthreads();
@@ -72,6 +73,10 @@ __global__ __launch_bounds__(256) void k_pred_logits(const uint8_t *__restrict__
         const unsigned long long m = __ballot(on);
         if (lane == 0) mask[blockIdx.x] = m;
     }
+}
+
+static auto logits_kernel(int rank) {
+    return llg_pred_wide(rank) ? k_pred_logits<PRED_MAXV_WIDE> : k_pred_logits<PRED_MAXV>;
 }
 
 // Masks from given logits (predictor.go:76-82 on its own).
@@ -176,7 +181,7 @@ int llg_pred_masks_enqueue(LlgDevice *d, LlgObject *wup, LlgObject *wout, LlgObj
     const int n_tiles = (ff + 63) / 64;
     const float *d_bias = bias ? reinterpret_cast<const float *>(bias->d) : nullptr;
     const size_t lds = (size_t)(((rank + 3) & ~3) + 64) * sizeof(float);
-    hipLaunchKernelGGL(k_pred_logits, dim3(n_tiles), dim3(256), lds, llg_dev_stream(d), wout->d,
+    hipLaunchKernelGGL(logits_kernel(rank), dim3(n_tiles), dim3(256), lds, llg_dev_stream(d), wout->d,
                        wout->stride, ff, rank, partial, d_bias, thr, (float *)nullptr, *mask_out);
     LLG_LAUNCH_CHECK(d, "pred_logits");
     return 0;
@@ -204,7 +209,7 @@ int llg_pred_logits_enqueue(LlgDevice *d, LlgObject *wout, LlgObject *bias, floa
     const int n_tiles = (ff + 63) / 64;
     const float *d_bias = bias ? reinterpret_cast<const float *>(bias->d) : nullptr;
     const size_t lds = (size_t)(((rank + 3) & ~3) + 64) * sizeof(float);
-    hipLaunchKernelGGL(k_pred_logits, dim3(n_tiles), dim3(256), lds, llg_dev_stream(d), wout->d,
+    hipLaunchKernelGGL(logits_kernel(rank), dim3(n_tiles), dim3(256), lds, llg_dev_stream(d), wout->d,
                        wout->stride, ff, rank, partial, d_bias, thr, d_logits, mask);
     LLG_LAUNCH_CHECK(d, "pred_logits");
     return llg_compact_enqueue(d, mask, n_tiles, d_active, d_n_active);

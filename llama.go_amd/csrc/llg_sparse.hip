@@ -482,13 +482,14 @@ constexpr int tf_dk() {
 }
 
 // The logit of row 16 w + l / 4 of the tile in every lane l of wavefront w
-// (the quad layout of load_wout_tile; the scalar layout for other ranks),
+// (the quad layout of load_wout_tile; the scalar layout for larger ranks),
 // the same sums as finish_logits.
-__device__ __forceinline__ float tile_logit(const WoutTile &t, const uint8_t *__restrict__ wout,
+template <int MV>
+__device__ __forceinline__ float tile_logit(const WoutTile<MV> &t, const uint8_t *__restrict__ wout,
                                             long long stride, int ff, int rank, int tile0,
                                             const float *hid) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (t.v) return wout_tile_dot(t, hid);
+    if (t.v) return wout_tile_dot(t, hid, rank);
     float mine = 0.0f;
     for (int r = 0; r < 16; r++) {
         const int i = tile0 + wave * 16 + r;
@@ -526,7 +527,8 @@ struct HidArgs {
     const float *a;          // predictor input
     uint64_t *slots;         // sync slots, after the epoch word at ctr
     const uint32_t *ctr;
-    int n_hid;               // predictor workgroups at the head of the grid
+    int n_hid;               // predictor workgroups at the head of the grid,
+    int rpw;                 // of this many hidden units each
     float *acc_out;          // optional: acc_out[i] += acc_add[i], i < acc_n
     const float *acc_add;
     int acc_n;
@@ -561,13 +563,12 @@ struct WoArgs {
 // past it the workgroup computes the missing units itself.
 #define HID_POLLS (1 << 16)
 
-// A predictor workgroup: RPW hidden units; wavefront s < LLG_PRED_SPLIT takes
+// A predictor workgroup of RPW hidden units: wavefront s < LLG_PRED_SPLIT takes
 // chunk s of each unit's WUp row (the sums of k_pred_hidden, the rows sharing
 // the loads of a), then every copy of the units' slots is written.
-template <int NW>
-__device__ __forceinline__ void tile_hid_role(const HidArgs &ha, int rank, float *sh) {
-    constexpr int RPW = NW / LLG_PRED_SPLIT;  // hidden units per workgroup
-    static_assert(RPW >= 1 && NW % LLG_PRED_SPLIT == 0, "whole units per workgroup");
+template <int RPW>
+__device__ __forceinline__ void tile_hid_units(const HidArgs &ha, int rank, float *sh) {
+    static_assert(RPW * LLG_SYNC_COPIES <= 512, "a thread per slot");
     // the epoch word as a vector load ahead of the row loads, waited on only
     // at the slot stores
     const uint32_t ctr = llg_epoch_get(ha.ctr);
@@ -595,6 +596,23 @@ __device__ __forceinline__ void tile_hid_role(const HidArgs &ha, int rank, float
     if (ha.acc_out)
         for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < ha.acc_n; i += ha.n_hid * blockDim.x)
             ha.acc_out[i] += ha.acc_add[i];
+}
+
+// ... of the count the launch chose (hid_units): NW / 8, twice, 4 or 8 times that.
+template <int NW, int MV>
+__device__ __forceinline__ void tile_hid_role(const HidArgs &ha, int rank, float *sh) {
+    constexpr int R = NW / LLG_PRED_SPLIT;
+    static_assert(R >= 1 && NW % LLG_PRED_SPLIT == 0, "whole units per workgroup");
+    if ((NW > 8 && MV <= PRED_MAXV) || ha.rpw == R)
+        tile_hid_units<R>(ha, rank, sh);
+    else if (ha.rpw == 2 * R)
+        tile_hid_units<2 * R>(ha, rank, sh);
+    else if constexpr (NW <= 8) {
+        if (ha.rpw == 4 * R)
+            tile_hid_units<4 * R>(ha, rank, sh);
+        else
+            tile_hid_units<8 * R>(ha, rank, sh);
+    }
 }
 
 // Hidden unit j of the predictor (ReLU'd, predictor.go:61) from the attention
@@ -801,7 +819,7 @@ __device__ __forceinline__ void tile_take_comb(float *hid, const WoArgs &wa, con
 // k_tile_reduce adds the partials in a fixed order, so the result is the
 // same on every run.
 // WO: the instance with Wo's workgroups at the head of the grid (k_tile_wo_ffn).
-template <int T, bool WO>
+template <int T, bool WO, int MV>
 __device__ __forceinline__ void tile_ffn_body(
     const uint8_t *__restrict__ wout, long long wstride, int ff, int rank,
     const float *__restrict__ partial, const float *__restrict__ bias, float thr,
@@ -811,7 +829,7 @@ __device__ __forceinline__ void tile_ffn_body(
     extern __shared__ float sh[];
     constexpr int TW = tf_tiles<T>(), NT = TW * TU, NTH = tf_threads<T>(), NW = NTH / 64;
     if ((int)blockIdx.x < ha.n_hid) {
-        tile_hid_role<NW>(ha, rank, sh);
+        tile_hid_role<NW, MV>(ha, rank, sh);
         return;
     }
     if constexpr (WO) {
@@ -837,7 +855,7 @@ __device__ __forceinline__ void tile_ffn_body(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int *tl = reinterpret_cast<int *>(wm + NW) + wave * NT;  // this wavefront's active list
     const int n0 = ti * NT, n1 = min(ff, n0 + NT);
-    WoutTile t;  // logits: wavefronts with neurons in the tile
+    WoutTile<MV> t;  // logits: wavefronts with neurons in the tile
     const bool lw = wave * 16 < n1 - n0;
     uint64_t hv0 = 0;
     uint32_t ctr = 0;
@@ -980,26 +998,26 @@ __device__ __forceinline__ void tile_ffn_body(
     }
 }
 
-template <int T>
+template <int T, int MV>
 __global__ __launch_bounds__(tf_threads<T>(), tf_threads<T>() / 256) void k_tile_ffn(
     const uint8_t *__restrict__ wout, long long wstride, int ff, int rank,
     const float *__restrict__ partial, const float *__restrict__ bias, float thr,
     const uint8_t *__restrict__ base, long long bstride, RowFmt f, const float *__restrict__ x,
     int act, unsigned long long *__restrict__ mask, float *__restrict__ part, int pstride,
     HidArgs ha) {
-    tile_ffn_body<T, false>(wout, wstride, ff, rank, partial, bias, thr, base, bstride, f, x, act,
+    tile_ffn_body<T, false, MV>(wout, wstride, ff, rank, partial, bias, thr, base, bstride, f, x, act,
                             mask, part, pstride, ha, WoArgs{});
 }
 
 // The same with Wo's workgroups (WoArgs) at the head of the grid.
-template <int T>
+template <int T, int MV>
 __global__ __launch_bounds__(tf_threads<T>(), tf_threads<T>() / 256) void k_tile_wo_ffn(
     const uint8_t *__restrict__ wout, long long wstride, int ff, int rank,
     const float *__restrict__ bias, float thr, const uint8_t *__restrict__ base,
     long long bstride, RowFmt f, const float *__restrict__ x, int act,
     unsigned long long *__restrict__ mask, float *__restrict__ part, int pstride, HidArgs ha,
     WoArgs wa) {
-    tile_ffn_body<T, true>(wout, wstride, ff, rank, nullptr, bias, thr, base, bstride, f, x, act,
+    tile_ffn_body<T, true, MV>(wout, wstride, ff, rank, nullptr, bias, thr, base, bstride, f, x, act,
                            mask, part, pstride, ha, wa);
 }
 
@@ -1606,8 +1624,26 @@ static size_t tile_lds_bytes(const RowFmt &f, int rank) {
     return xs_bytes(f) + (size_t)(((rank + 3) & ~3) + NT + NW + NW * NT) * 4;
 }
 
+// Hidden units per predictor workgroup: the fewest (the shortest hand-off) with
+// which the predictor and the tile workgroups, one per CU at a time (each takes
+// a CU's registers), need no more rounds of the chip than with the most, so
+// that no tile waits for a predictor workgroup's CU.  Past 8 rows' loads in a
+// lane the registers spill (Q4_0's 1024 threads: past 4, and its narrow form's
+// ranks do not need more than 2).  Measured, Q8_0:
+// 4096 x 14336 at rank 256, 1 -> 8 units: 480 -> 256 workgroups, one round;
+// 4544 x 18176 at rank 128, two rounds either way: 1 unit 19.1, 8 units 21.3 us.
 template <int T>
-static void launch_fused(hipStream_t st, LlgObject *wout, const float *partial,
+static int hid_units(int cus, int rank, int n_parts, bool wide) {
+    constexpr int NW = tf_threads<T>() / 64, R = NW / LLG_PRED_SPLIT;
+    const int RM = NW <= 8 ? 8 * R : wide ? 2 * R : R;
+    auto rounds = [&](int r) { return ((rank + r - 1) / r + n_parts + cus - 1) / cus; };
+    int r = R;
+    while (r < RM && rounds(r) > rounds(RM)) r *= 2;
+    return r;
+}
+
+template <int T>
+static void launch_fused(hipStream_t st, int cus, LlgObject *wout, const float *partial,
                          const float *bias, float thr, LlgObject *b, const float *x, int act,
                          unsigned long long *mask, float *part, int32_t *n_active, float *out,
                          bool accumulate, float2 *stats, HidArgs ha, WoArgs wa) {
@@ -1617,7 +1653,11 @@ static void launch_fused(hipStream_t st, LlgObject *wout, const float *partial,
     const int pstride = f.nb * 32;
     constexpr int NT = tf_tiles<T>() * TU, NW = tf_threads<T>() / 64;
     const int n_parts = (ff + NT - 1) / NT;  // tile workgroups, one partial row each
-    if (ha.slots && ha.wup) ha.n_hid = (rank + NW / LLG_PRED_SPLIT - 1) / (NW / LLG_PRED_SPLIT);
+    const bool wide = llg_pred_wide(rank);
+    if (ha.slots && ha.wup) {
+        ha.rpw = hid_units<T>(cus, rank, n_parts, wide);
+        ha.n_hid = (rank + ha.rpw - 1) / ha.rpw;
+    }
     size_t lds = tile_lds_bytes<T>(f, rank);
     if (wa.w) {
         wa.n_comb = (rank + NW - 1) / NW;
@@ -1625,11 +1665,11 @@ static void launch_fused(hipStream_t st, LlgObject *wout, const float *partial,
         lds = std::max(lds, (size_t)wa.f.nb * XS_STRIDE * 4);
     }
     if (wa.w)
-        hipLaunchKernelGGL((k_tile_wo_ffn<T>), dim3(wa.n_comb + n_parts + wa.n_wo), dim3(tf_threads<T>()), lds,
+        hipLaunchKernelGGL((wide ? k_tile_wo_ffn<T, PRED_MAXV_WIDE> : k_tile_wo_ffn<T, PRED_MAXV>), dim3(wa.n_comb + n_parts + wa.n_wo), dim3(tf_threads<T>()), lds,
                            st, wout->d, wout->stride, ff, rank, bias, thr, b->d, b->stride, f, x,
                            act, mask, part, pstride, ha, wa);
     else
-        hipLaunchKernelGGL((k_tile_ffn<T>), dim3(ha.n_hid + n_parts), dim3(tf_threads<T>()), lds,
+        hipLaunchKernelGGL((wide ? k_tile_ffn<T, PRED_MAXV_WIDE> : k_tile_ffn<T, PRED_MAXV>), dim3(ha.n_hid + n_parts), dim3(tf_threads<T>()), lds,
                            st, wout->d, wout->stride, ff, rank, partial, bias, thr, b->d,
                            b->stride, f, x, act, mask, part, pstride, ha);
     uint32_t *ctr = ha.slots ? const_cast<uint32_t *>(ha.ctr) : nullptr;
@@ -1668,19 +1708,19 @@ static int fused_tail(LlgDevice *d, LlgObject *wout, LlgObject *bias, LlgObject 
     hipStream_t st = llg_dev_stream(d);
     switch (f.type) {
     case LLG_TYPE_Q4_0:
-        launch_fused<LLG_TYPE_Q4_0>(st, wout, partial, d_bias, thr, b, d_x, act, mask, part,
+        launch_fused<LLG_TYPE_Q4_0>(st, llg_cu_count(d), wout, partial, d_bias, thr, b, d_x, act, mask, part,
                                     d_n_active, d_out, accum, d_stats, ha, wa);
         break;
     case LLG_TYPE_Q8_0:
-        launch_fused<LLG_TYPE_Q8_0>(st, wout, partial, d_bias, thr, b, d_x, act, mask, part,
+        launch_fused<LLG_TYPE_Q8_0>(st, llg_cu_count(d), wout, partial, d_bias, thr, b, d_x, act, mask, part,
                                     d_n_active, d_out, accum, d_stats, ha, wa);
         break;
     case LLG_TYPE_F16:
-        launch_fused<LLG_TYPE_F16>(st, wout, partial, d_bias, thr, b, d_x, act, mask, part,
+        launch_fused<LLG_TYPE_F16>(st, llg_cu_count(d), wout, partial, d_bias, thr, b, d_x, act, mask, part,
                                    d_n_active, d_out, accum, d_stats, ha, wa);
         break;
     case LLG_TYPE_F32:
-        launch_fused<LLG_TYPE_F32>(st, wout, partial, d_bias, thr, b, d_x, act, mask, part,
+        launch_fused<LLG_TYPE_F32>(st, llg_cu_count(d), wout, partial, d_bias, thr, b, d_x, act, mask, part,
                                    d_n_active, d_out, accum, d_stats, ha, wa);
         break;
     default:
