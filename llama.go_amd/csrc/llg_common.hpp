@@ -1011,6 +1011,21 @@ uint64_t *llg_dev_mvslots(LlgDevice *d, size_t bytes, int *rc);
 // clears its slots, then computes each handed-over value itself and uses its
 // own, so that a test can compare the fallback path with the slots bit for bit.
 int llg_dev_check(LlgDevice *d);
+// Pinned staging of the small host-buffer calls: at least `bytes` of the
+// handle's pinned host memory (at most LLG_STAGE_MAX, freed with the handle),
+// or null (too large, or no memory: the caller copies from pageable memory
+// instead).  A call that uses it ends with a stream synchronisation, so the
+// next call finds it free.  llg_stage_in copies `bytes` from the staging area's
+// offset `off` to the device, llg_stage_out back; with list, the first
+// min(*list_n, list_cap) entries of it to offset list_off as well.  Kernels do
+// the copies: a hipMemcpyAsync of pageable memory costs 8 - 15 us each.
+// dst / src and off are 16-byte aligned, their spans whole 16-byte units.
+#define LLG_STAGE_MAX ((size_t)1 << 20)
+uint8_t *llg_host_stage(LlgDevice *d, size_t bytes);
+int llg_stage_in(LlgDevice *d, void *dst, size_t off, size_t bytes);
+int llg_stage_out(LlgDevice *d, const void *src, size_t off, size_t bytes,
+                  const int32_t *list = nullptr, const int32_t *list_n = nullptr, int list_cap = 0,
+                  size_t list_off = 0);
 // Copy host -> device workspace slot / device -> host, on the stream.
 int llg_h2d(LlgDevice *d, void *dst, const void *src, size_t bytes);
 int llg_d2h(LlgDevice *d, void *dst, const void *src, size_t bytes);

@@ -7,6 +7,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 #include <unordered_map>
 
@@ -25,6 +26,9 @@ struct LlgDevice {
     uint8_t *sync = nullptr;  // LLG_SYNC_BYTES, zeroed at allocation
     uint64_t *mvslots = nullptr;  // chunked matvecs' hand-off slots, zero between calls
     size_t mvslots_bytes = 0;
+    uint8_t *stage = nullptr;  // pinned host memory of the host-buffer calls
+    uint8_t *stage_dev = nullptr;  // its device address
+    size_t stage_bytes = 0;
     int check_handoff = 0;  // LLG_CHECK_HANDOFF at creation (llg_dev_check)
     std::string last_error;
     bool tearing_down = false;  // llg_hip_free: every object is freed in one sweep
@@ -96,6 +100,68 @@ uint64_t *llg_dev_mvslots(LlgDevice *d, size_t bytes, int *rc) {
     d->mvslots_bytes = want;
     return d->mvslots;
 }
+uint8_t *llg_host_stage(LlgDevice *d, size_t bytes) {
+    if (bytes > LLG_STAGE_MAX) return nullptr;
+    if (bytes <= d->stage_bytes) return d->stage;
+    size_t want = 64 << 10;
+    while (want < bytes) want *= 2;
+    if (d->stage) {
+        hipStreamSynchronize(d->stream);
+        hipHostFree(d->stage);
+        d->stage = nullptr;
+        d->stage_bytes = 0;
+    }
+    void *p = nullptr, *dp = nullptr;
+    if (hipHostMalloc(&p, want, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (hipHostGetDevicePointer(&dp, p, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        hipHostFree(p);
+        return nullptr;
+    }
+    d->stage = static_cast<uint8_t *>(p);
+    d->stage_dev = static_cast<uint8_t *>(dp);
+    d->stage_bytes = want;
+    return d->stage;
+}
+
+// Copies n16 16-byte units (a workgroup's loads are whole lines over the
+// link), then, with list, list[0 .. min(*list_n, list_cap)) to list_dst.
+__global__ __launch_bounds__(256) void k_stage_copy(const uint4 *__restrict__ src,
+                                                    uint4 *__restrict__ dst, int n16,
+                                                    const int32_t *__restrict__ list,
+                                                    const int32_t *__restrict__ list_n,
+                                                    int list_cap, int32_t *__restrict__ list_dst) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+    for (int i = t; i < n16; i += step) dst[i] = src[i];
+    if (!list) return;
+    const int n = min(max(*list_n, 0), list_cap);
+    for (int i = t; i < n; i += step) list_dst[i] = list[i];
+}
+
+static int stage_copy(LlgDevice *d, const void *src, void *dst, size_t bytes, const int32_t *list,
+                      const int32_t *list_n, int list_cap, int32_t *list_dst) {
+    const int n16 = (int)((bytes + 15) / 16);
+    const int grid = std::max(1, std::min(64, (std::max(n16, list ? list_cap / 4 : 0) + 255) / 256));
+    hipLaunchKernelGGL(k_stage_copy, dim3(grid), dim3(256), 0, d->stream,
+                       static_cast<const uint4 *>(src), static_cast<uint4 *>(dst), n16, list, list_n,
+                       list_cap, list_dst);
+    LLG_LAUNCH_CHECK(d, "stage copy");
+    return 0;
+}
+
+int llg_stage_in(LlgDevice *d, void *dst, size_t off, size_t bytes) {
+    return stage_copy(d, d->stage_dev + off, dst, bytes, nullptr, nullptr, 0, nullptr);
+}
+
+int llg_stage_out(LlgDevice *d, const void *src, size_t off, size_t bytes, const int32_t *list,
+                  const int32_t *list_n, int list_cap, size_t list_off) {
+    return stage_copy(d, src, d->stage_dev + off, bytes, list, list_n, list_cap,
+                      reinterpret_cast<int32_t *>(d->stage_dev + list_off));
+}
+
 hipStream_t llg_dev_stream(LlgDevice *d) { return d->stream; }
 int llg_dev_check(LlgDevice *d) { return d->check_handoff; }
 int llg_device_id(LlgDevice *d) { return d->device; }
@@ -339,6 +405,7 @@ void llg_hip_free(LlgHipDevice h) {
     if (d->ws) hipFree(d->ws);
     if (d->sync) hipFree(d->sync);
     if (d->mvslots) hipFree(d->mvslots);
+    if (d->stage) hipHostFree(d->stage);
     hipStreamDestroy(d->stream);
     delete d;
 }
